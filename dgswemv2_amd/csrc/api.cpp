@@ -413,24 +413,25 @@ struct Engine final : EngineBase {
                 return RKDG_ERR_HIP;
         }
         if (!M.sp_vol.empty() && (!upload(sp_vol, M.sp_vol) || !upload(sp_edge, M.sp_edge))) return RKDG_ERR_HIP;
-        std::vector<double> fast_geom, fast_edge;
+        std::vector<double> fast_geom, fast_edge, fast_gmn2;
         const bool scaled = fast && rkdg::scaled_geometry<Real>(M.p);
         if (scaled) {
-            fast_geom = M.geom, fast_edge = M.egeom;
+            fast_geom = M.geom, fast_edge = M.egeom, fast_gmn2 = M.gmn2;
             const size_t n = M.nedge;
             for (size_t i = 0; i < n; ++i) {
                 const double hs = 0.5 * M.egeom[2 * n + i];
                 fast_edge[i] = hs * M.egeom[i], fast_edge[n + i] = hs * M.egeom[n + i], fast_edge[2 * n + i] = hs;
             }
+            fast_geom.resize(6 * ne);
             for (size_t e = 0; e < ne; ++e) {
                 const double adet = M.geom[4 * ne + e];
                 for (int c = 0; c < 4; ++c) fast_geom[c * ne + e] = M.geom[c * ne + e] * adet;
-                fast_geom[4 * ne + e] = 1.0 / adet;
+                fast_geom[4 * ne + e] = 1.0 / adet, fast_geom[5 * ne + e] = adet, fast_gmn2[e] *= adet;
             }
         }
         if (!upload(bath, M.bath) || !upload(geom, scaled ? fast_geom : M.geom) ||
             !upload(egeom, scaled ? fast_edge : M.egeom) || !upload(vxy, M.vxy) ||
-            !upload(gmn2, M.gmn2) || !upload(famp, M.famp) || !upload(fphase, M.fphase) ||
+            !upload(gmn2, scaled ? fast_gmn2 : M.gmn2) || !upload(famp, M.famp) || !upload(fphase, M.fphase) ||
             !upload(levee_gp, M.levee_gp) || !upload(nb, M.nb) ||
             !upload(edge, M.edge) || !upload(eforce, M.eforce) || !upload(meta, M.meta) ||
             !upload(neighbor, M.neighbor) || !upload(bath_vrtx, M.bath_vrtx))

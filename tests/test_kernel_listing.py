@@ -68,3 +68,28 @@ def test_no_copy_at_a_join_before_its_lanes_are_back(objects):
             if hits:
                 bad[_short(name)] = hits
     assert seen >= 36 and not bad, bad
+
+
+def test_registers_of_the_fast_stage(objects):
+    """(registers, accumulation registers) at most: 128, 168 and 256 are four, three and two waves a SIMD."""
+    limit = {("double", 1, False): 168, ("double", 2, False): 256, ("double", 1, True): 256, ("double", 2, True): 256,
+             ("float", 2, False): 128, ("float", 2, True): 168, ("float", 3, False): 256, ("float", 3, True): 256,
+             ("float", 1, False): 96, ("float", 1, True): 104}
+    seen, over = set(), {}
+    for obj in objects:
+        notes = subprocess.run([f"{LLVM}/llvm-readelf", "--notes", obj], check=True, capture_output=True, text=True).stdout
+        for k in re.split(r"\n  - \.agpr_count:", notes)[1:]:
+            sym = re.search(r"\.symbol:\s*'?([\w.]+)'?", k).group(1)
+            name = subprocess.run(["c++filt", sym.replace(".kd", "")], capture_output=True, text=True).stdout
+            m = re.search(r"stage_kernel(_persistent)?<(double|float), (\d), (\w+), false, true, (\w+)>", name)
+            if not m or (m.group(1) and m.group(5) == "false"):
+                continue
+            key = (m.group(2), int(m.group(3)), bool(m.group(1)))
+            if key not in limit:
+                continue
+            agpr = int(k.split("\n")[0])
+            vgpr = int(re.search(r"\.vgpr_count:\s*(\d+)", k).group(1))
+            seen.add(m.group(0))
+            if agpr or vgpr > limit[key]:
+                over[m.group(0)] = (vgpr, agpr)
+    assert len(seen) == 5 * 4 + 5 * 2 and not over, (len(seen), over)

@@ -31,7 +31,7 @@ __device__ __forceinline__ f32x4 mfma(const bf16x8& a, const bf16x8& b, const f3
 
 __device__ __forceinline__ float bf16_to_float(__bf16 b) { return (float)b; }
 
-// max(x, 0) in one instruction (v_med3_f32); fmaxf would also canonicalise NaNs
+// max(x, 0) in one instruction (v_med3_f32), 0 for a NaN; fmaxf would also canonicalise
 __device__ __forceinline__ float relu(float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, 3.40282347e38f); }
 
 // One hidden layer of 16 elements: D = W B (+ bias), W packed [mt][ks] (A operands), B in two
@@ -54,13 +54,16 @@ __device__ __forceinline__ bf16x8 pack8(const f32x4& a, const f32x4& b) {
     return __builtin_shufflevector(__builtin_convertvector(a, bf16x4), __builtin_convertvector(b, bf16x4), 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-// relu and repack D of M-tiles (0, 1) and (2, 3) as the B operands of the next layer's K-steps.  Rounding
-// to bf16 keeps the sign, so the relu runs on the packed bits: a negative bf16 is a negative int16.
+// relu and repack D of M-tiles (0, 1) and (2, 3) as the B operands of the next layer's K-steps.  The relu comes
+// before the rounding: a value that is no number counts as zero, and a maximum on the packed bits would keep it.
 __device__ __forceinline__ void relu_pack(const f32x4 (&acc)[4], bf16x8& b0, bf16x8& b1) {
-    typedef short s16x8 __attribute__((ext_vector_type(8)));
-    const s16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-    b0 = __builtin_bit_cast(bf16x8, __builtin_elementwise_max(__builtin_bit_cast(s16x8, pack8(acc[0], acc[1])), zero));
-    b1 = __builtin_bit_cast(bf16x8, __builtin_elementwise_max(__builtin_bit_cast(s16x8, pack8(acc[2], acc[3])), zero));
+    f32x4 r[4];
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) r[mt][jj] = relu(acc[mt][jj]);
+    b0 = pack8(r[0], r[1]);
+    b1 = pack8(r[2], r[3]);
 }
 
 // as relu_pack, for back-propagated values masked by the forward activations (bf16 > 0)

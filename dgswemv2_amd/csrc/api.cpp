@@ -544,14 +544,14 @@ struct Engine final : EngineBase {
         return e;
     }
     // learned form: the gate writes the troubled (gate) flags and the list of open elements; the limit
-    // pass runs over that list.  bary: the barycentres are written anew by the check kernel first.
+    // pass runs over that list.  bary: the gate writes the barycentres, too, from the modes that it reads.
     hipError_t learned_limiter(const rkdg::LimiterArgs<Real>& L, bool bary) {
         rkdg::GateArgs<Real> G = gate_args(L);
         G.wpack = ind_pack, G.vec = ind_vec, G.flag = troubled;
         G.limited = limited, G.list = ind_list, G.list_count = ind_count, G.list_cap = rkdg::gate_grid(M.ne).cap;
         if (cap_on) G.logit = cap_logit;
-        hipError_t e = bary ? rkdg::launch_limiter_check<Real>(M.p, L, true, stream, block) : hipSuccess;
-        if (e == hipSuccess) e = rkdg::launch_gate<Real>(M.p, G, true, stream);
+        if (bary) G.baryctr = baryctr;
+        hipError_t e = rkdg::launch_gate<Real>(M.p, G, true, stream);
         if (e == hipSuccess && (ind_judge || cap_on)) {
             rkdg::JudgeArgs J = judge_args();
             J.flag = troubled;
@@ -652,16 +652,17 @@ struct Engine final : EngineBase {
     bool gate_fused() const { return ind_on && ind_state && !ind_judge && !cap_on; }
     rkdg_status stage() override {
         const bool fused = gate_fused();
-        rkdg_status r = begin(fused);
+        rkdg_status r = begin(fused, !fused);
         return r == RKDG_OK ? finish(false, fused) : r;
     }
-    rkdg_status stage_begin() override { return begin(false); }
-    // the state may have changed since the stage kernel (a halo exchange): new barycentres
+    // the state may change between the stage kernel and the limiter (a halo exchange), so the limiter's first
+    // launch writes the barycentres
+    rkdg_status stage_begin() override { return begin(false, false); }
     rkdg_status stage_finish() override { return finish(true, false); }
     unsigned long long mid_key = 0;  // stage_key of the stage begun
     bool mid_tm = false;
 
-    rkdg_status begin(bool fused) {
+    rkdg_status begin(bool fused, bool bary) {
         if (mid_stage) return fail("stage_begin twice without stage_finish", hipErrorInvalidValue), RKDG_ERR_ARG;
         rkdg::Stepper& st = M.stepper;
         const int s = st.stage, ns = st.nstages;
@@ -701,7 +702,7 @@ struct Engine final : EngineBase {
         A.problem = M.prm.problem;
         for (int i = 0; i < 4; ++i) A.pparam[i] = M.prm.problem_param[i];
         A.h_o = M.h_o, A.h_thr = M.h_thr;
-        A.baryctr = M.prm.slope_limiting && !fused ? baryctr : nullptr;
+        A.baryctr = M.prm.slope_limiting && bary ? baryctr : nullptr;
         A.nan_check = (M.prm.slope_limiting && !ind_on) ? 0 : 1;  // the gated limiter scans only what it limits
         A.nan_key = d_nan;
         A.stage_key = (unsigned long long)st.step * ns + s;

@@ -198,6 +198,11 @@ __global__ void __launch_bounds__(kGateBlock) __attribute__((amdgpu_waves_per_eu
                     const Real val = in.val[9 * k + 3 * v + i];
                     x[9 * k + 3 * v + i] = (float)(i == 0 ? val - in.val[3 * v] : val);
                 }
+        if constexpr (MLP && !LIMIT)
+            if (G.baryctr && valid && in.wet[0])
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    stc(G.baryctr, ne, k, e, barycentre((double)in.val[3 * k], (double)in.val[3 * k + 1], (double)in.val[3 * k + 2]));
         const bool okw = (in.wet[0] & in.wet[1] & in.wet[2] & in.wet[3]) != 0;
         // physical scales; a variation at or below 1e-16 of its scale carries no shape
         float h = (float)((double)in.val[0] + in.bath);

@@ -114,6 +114,7 @@ struct GateArgs {
     float* logit;             // [ne] or null
     float* feat;              // [36][ne] or null
     uint8_t* ok;              // [ne] element and neighbours wet, or null
+    double* baryctr;          // [3][ne] barycentre values of wet elements for the limit pass, or null, MLP only
     uint8_t* limited;         // [3][ne] cleared (the limit pass sets it where it writes), MLP only
     int* list;                // elements whose gate is open: wave w's in list[w cap ..], MLP only
     int* list_count;          // [waves] how many each wave found, MLP only

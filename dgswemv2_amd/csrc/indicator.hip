@@ -80,13 +80,6 @@ __device__ __forceinline__ void mask_pack(const f32x4 (&acc)[4], const bf16x8& h
 
 __device__ __forceinline__ uint16_t bits(__bf16 b) { return __builtin_bit_cast(uint16_t, b); }
 
-// Orders a wave's LDS writes before its later LDS reads of other lanes' data (no work-group barrier).
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // store a packed pair (neurons of M-tiles 2 ks, 2 ks + 1) as rows of a [64][ld] bf16 array
 __device__ __forceinline__ void store_rows(uint16_t* dst, long long ld, int col, int g, const bf16x8& b0,
                                            const bf16x8& b1) {

@@ -9,7 +9,7 @@
 //   sl_check_element    - the KXRCF-style indicator I of check_trouble (swe_trouble_check.hpp:13-104),
 //                         written as the seed set (and, for a state that changed after its stage
 //                         kernel, the barycentres);
-//   sl_spread_seed      - the six neighbour-dilation passes (:106-115) of one seed;
+//   sl_spread_seeds     - the six neighbour-dilation passes (:106-115), by the limit kernel;
 //   sl_limit_core       - slope_limiting_kernel (swe_CS_slope_limiter.hpp:88-189) reading the
 //                         neighbours' barycentres, then the NaN scan.
 // The limit pass never reads the troubled flags: they are an output.
@@ -137,26 +137,6 @@ RKDG_HD RKDG_FORCE_INLINE inline void sl_check_element(const LimiterArgs<Real>& 
     }
     L.seed[e] = seed;
     L.troubled[e] = seed;
-}
-
-// One lane's share of the dilation of seed e: six passes over interior neighbours mark the elements
-// up to five steps away.  Lane l < 48 follows one walk of five steps that never turns back (three
-// first steps, then one of two); the 48 walks together visit the whole ball.  A walk ends at a
-// boundary and at another seed, whose own walks cover everything beyond it.  Writes of 1 only.
-RKDG_HD inline void sl_spread_seed(int ne, const int* neighbor, const uint8_t* seed, uint8_t* troubled, int e, int l) {
-    int prev = -1, cur = e, turns = l >> 4;
-    for (int step = 0; step < 5; ++step) {
-        int next = -1, skip = turns;
-        for (int k = 0; k < 3; ++k) {
-            const int n = neighbor[(size_t)k * ne + cur];
-            if (n == prev && step > 0) continue;
-            if (skip-- == 0) next = n;
-        }
-        if (next < 0 || seed[next]) return;
-        troubled[next] = 1;
-        prev = cur, cur = next;
-        turns = (l >> step) & 1;
-    }
 }
 
 RKDG_HD inline void mv3(const double A[3][3], const double* x, double* y) {

@@ -204,9 +204,10 @@ struct Engine final : EngineBase {
         if (ramp_tab_h) hipHostFree(ramp_tab_h);
         for (Staging& l : staging)
             for (int i = 0; i < 2; ++i) {
-                if (l.buf[i]) hipHostFree(l.buf[i]);
+                if (l.buf[i] && !l.of_slab) hipHostFree(l.buf[i]);
                 if (l.ev[i]) hipEventDestroy(l.ev[i]);
             }
+        if (slab) hipHostFree(slab);
         if (nan_h) hipHostFree(nan_h);
     }
 
@@ -216,15 +217,29 @@ struct Engine final : EngineBase {
     // of the whole state into a freshly allocated host vector.  A large state is read by several host
     // threads, each with a pair of its own (144 MB: 10.2 ms by one, 5.0 by eight; 9 MB by one 410 us, by
     // two 425).  The first buffer's tail holds flags.
-    static constexpr size_t kPinBytes = size_t(1) << 20, kFlagBytes = size_t(256) << 10, kReaderBytes = size_t(8) << 20;
+    static constexpr size_t kPinBytes = size_t(1) << 20, kFlagBytes = size_t(256) << 10, kReaderBytes = size_t(8) << 20,
+                            kWriteBytes = size_t(4) << 20;
     static constexpr int kReaders = 8;
     struct Staging {
         void* buf[2] = {nullptr, nullptr};
         hipEvent_t ev[2] = {nullptr, nullptr};
+        bool of_slab = false;
     };
     Staging staging[kReaders];
+    void* slab = nullptr;  // the further readers' buffers in one piece, allocated by the first reading that needs any
+    size_t slab_bytes = 0;
     unsigned long long* nan_h = nullptr;  // the NaN record, pinned
     hipError_t ensure_pinned(int n) {
+        if (n > 1 && !slab) {
+            const size_t bytes = (size_t)(n - 1) * 2 * kPinBytes;
+            const hipError_t e = hipHostMalloc(&slab, bytes, hipHostMallocDefault);
+            if (e != hipSuccess) return slab = nullptr, e;
+            slab_bytes = bytes;
+            for (int k = 1; k < n; ++k) {
+                staging[k].of_slab = true;
+                for (int i = 0; i < 2; ++i) staging[k].buf[i] = static_cast<char*>(slab) + (2 * (size_t)(k - 1) + i) * kPinBytes;
+            }
+        }
         for (int k = 0; k < n; ++k)
             for (int i = 0; i < 2; ++i) {
                 Staging& l = staging[k];
@@ -356,21 +371,25 @@ struct Engine final : EngineBase {
     }
     // host -> device: chunk c is converted into buffer c % 2 once that buffer's previous copy
     // (chunk c - 2, or a copy of an earlier call still in flight) has completed, then copied
-    // while chunk c + 1 is converted; the copies are asynchronous on the context's stream
+    // while chunk c + 1 is converted; the copies are asynchronous on the context's stream.  Where readings of
+    // a large state have left a slab, its chunks are larger: a copy costs some 3 us beyond its bytes (144 MB by
+    // 1 MB 5.2 ms, by 4 MB 4.7; 72 MB 2.66 and 2.33).
     hipError_t write_state(Real* dev, const double* in, size_t n) {
         hipError_t e = ensure_pinned(1);
         if (e != hipSuccess) return e;
-        Staging& l = staging[0];
-        const size_t per = kPinBytes / sizeof(Real), nch = (n + per - 1) / per;
+        const bool large = slab_bytes >= 2 * kWriteBytes && n * sizeof(Real) > 2 * kWriteBytes;
+        hipEvent_t* const ev = large ? staging[1].ev : staging[0].ev;
+        void* const buf[2] = {large ? slab : staging[0].buf[0], large ? static_cast<char*>(slab) + kWriteBytes : staging[0].buf[1]};
+        const size_t per = (large ? kWriteBytes : kPinBytes) / sizeof(Real), nch = (n + per - 1) / per;
         for (size_t c = 0; c < nch && e == hipSuccess; ++c) {
             const size_t off = c * per, cnt = std::min(per, n - off);
-            e = hipEventSynchronize(l.ev[c & 1]);  // returns at once for an event never recorded
-            Real* dst = static_cast<Real*>(l.buf[c & 1]);
+            e = hipEventSynchronize(ev[c & 1]);  // returns at once for an event never recorded
+            Real* dst = static_cast<Real*>(buf[c & 1]);
             if (e == hipSuccess) {
                 for (size_t i = 0; i < cnt; ++i) dst[i] = (Real)in[off + i];
                 e = hipMemcpyAsync(dev + off, dst, cnt * sizeof(Real), hipMemcpyHostToDevice, stream);
             }
-            if (e == hipSuccess) e = hipEventRecord(l.ev[c & 1], stream);
+            if (e == hipSuccess) e = hipEventRecord(ev[c & 1], stream);
         }
         return e;
     }

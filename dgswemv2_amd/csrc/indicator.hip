@@ -116,6 +116,9 @@ __device__ __forceinline__ void store_rows(uint16_t* dst, long long ld, int col,
 // are read for every pair of groups: as 96 registers a lane they left one or two waves per SIMD and
 // every wave fetched its own 24 KB.  Tried: one entity of an element per lane, so that the features
 // are the operands without LDS (40 % more vector instructions, 29 us against 26 us at 500k triangles).
+// Three waves a SIMD are asked for.  With LIMIT that spills: 20 registers to 84 B of scratch in FP64, 2 to 12 B
+// in FP32.  FP64 with two waves and no scratch, gate and limit pass: 500k triangles 49.7 us against 45.5 with
+// 3 % open, 53.7 against 51.6 with all open; 45k triangles 15.4 against 17.6 and 14.0 against 17.2.
 constexpr int kGateRow = 32 + 8;   // bf16 per element row in LDS: slots 0..7 of the four entities, then the
                                    // four slots 8 (and padding to 80 B)
 constexpr int kGateBlock = 256;

@@ -108,7 +108,7 @@ __device__ __forceinline__ void store_rows(uint16_t* dst, long long ld, int col,
 // LIMIT (p = 1): the limit pass of the open elements in the same launch.  The state is read from one
 // array and written, limited or as it was, to another, so no lane sees a limited neighbour; the
 // barycentres come from the modes phase 1 read.  Saves the list, the barycentre array, a second read of the
-// open elements and a launch.  Gate and limit pass together: 500k triangles with 2 % open 38 -> 31 us (one wave
+// open elements and a launch.  Gate and limit pass together: 500k triangles with 4 % open 38 -> 31 us (one wave
 // limited a whole list segment before: 61 us with most of them open, now 43 us), 45k triangles 14.5 -> 12 us.
 //
 // Bound by vector issue, some 800 instructions a tile and some 1,100 more for a tile with open elements,

@@ -1,14 +1,15 @@
 // Cockburn-Shu slope limiter and trouble check, per element (FP64 arithmetic in every form).
 //
-// The arithmetic is FP64 without fused multiply-adds in every form (each function turns contraction
-// off, whatever the translation unit's setting), so a limiter decision depends only on the state.
+// The arithmetic is FP64 and not contracted in any form (each function turns contraction off, whatever the
+// translation unit's setting), so a limiter decision depends only on the state.  The one place with fused
+// multiply-adds, written out, is the write-back of an FP32 state (sl_decide<true>).
 //
 // CS_slope_limiter_serial (problem_slope_limiter/swe_CS_sl_serial.hpp:9-23) as kernels:
 //   barycentres         - of the linear part (slope_limiting_prepare_element_kernel,
-//                         swe_CS_slope_limiter.hpp:8-20), written by the stage kernel;
+//                         swe_CS_slope_limiter.hpp:8-20), written by the stage kernel, or by the limiter's
+//                         first launch where the state may change in between (a stage in two calls);
 //   sl_check_element    - the KXRCF-style indicator I of check_trouble (swe_trouble_check.hpp:13-104),
-//                         written as the seed set (and, for a state that changed after its stage
-//                         kernel, the barycentres);
+//                         written as the seed set;
 //   sl_spread_seeds     - the six neighbour-dilation passes (:106-115), by the limit kernel;
 //   sl_limit_core       - slope_limiting_kernel (swe_CS_slope_limiter.hpp:88-189) reading the
 //                         neighbours' barycentres, then the NaN scan.
@@ -52,7 +53,7 @@ struct LimiterArgs {
 
 // BARY: writes the barycentres too.  Only a wet element can be a seed; its own data and then its
 // neighbours' are read together (two round trips; 190 B an element at p = 1 in FP64: 500k triangles
-// 24.7 -> 20 us, 33k triangles 5.5 -> 4.5 us).
+// 24.7 -> 16.6 us, 33k triangles 5.5 -> 4 us).
 template <typename Real, int P, bool BARY>
 RKDG_HD RKDG_FORCE_INLINE inline void sl_check_element(const LimiterArgs<Real>& L, const FaceTables<Real>& FT, int e) {
 #pragma clang fp contract(off)
